@@ -1,6 +1,6 @@
 // Measurement and test hooks (include/strasgpt_kbench.h): the calibration
-// copy for HBM traffic counters, the sustained matrix-core rate probe, and
-// the expert kernels' MXFP4 decode on host-supplied blocks.
+// copy for HBM traffic counters, the sustained matrix-core rate probe, the
+// expert kernels' MXFP4 decode on host-supplied blocks, and the launch rules.
 #include "device_common.h"
 #include "hip_check.h"
 #include "kernels.h"
@@ -152,6 +152,13 @@ extern "C" int strasgpt_kbench_mfma(int random_operands, int waves_per_simd, int
   HIP_CHECK(hipEventDestroy(e1));
   HIP_CHECK(hipFree(out));
   HIP_CHECK(hipStreamDestroy(s));
+  return 0;
+}
+
+extern "C" int strasgpt_kbench_gemm_splits(int M, int N, int K, int* qkv_splits, int* splits) {
+  if (M < 1 || N < 1 || K < 32 || !qkv_splits || !splits) return -1;
+  *qkv_splits = sg::gemm_qkv_splits(M, N, K, (size_t)-1);
+  *splits = sg::gemm_splits(M, N, K);
   return 0;
 }
 
