@@ -50,10 +50,10 @@ int strasgpt_kbench_mfma(int random_operands, int waves_per_simd, int iters, int
 int strasgpt_kbench_sort_desc(const uint32_t* keys, int n, uint32_t* keys_out, int32_t* index_out);
 
 /* The split-K factors that the prefill takes for M rows times an N x K
- * projection (host arithmetic, no GPU needed): qkv_splits as the QKV
- * projection of a workspace without bound, splits as the O or down
- * projection. */
-int strasgpt_kbench_gemm_splits(int M, int N, int K, int* qkv_splits, int* splits);
+ * projection in a precision of transformer_set_prefill_precision (host
+ * arithmetic, no GPU needed): qkv_splits as the QKV projection with a
+ * workspace without bound, splits as the O or down projection. */
+int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, int* qkv_splits, int* splits);
 
 #ifdef __cplusplus
 }

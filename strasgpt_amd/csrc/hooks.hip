@@ -155,10 +155,10 @@ extern "C" int strasgpt_kbench_mfma(int random_operands, int waves_per_simd, int
   return 0;
 }
 
-extern "C" int strasgpt_kbench_gemm_splits(int M, int N, int K, int* qkv_splits, int* splits) {
-  if (M < 1 || N < 1 || K < 32 || !qkv_splits || !splits) return -1;
-  *qkv_splits = sg::gemm_qkv_splits(M, N, K, (size_t)-1);
-  *splits = sg::gemm_splits(M, N, K);
+extern "C" int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, int* qkv_splits, int* splits) {
+  if (M < 1 || N < 1 || K < 32 || precision < 0 || precision > 1 || !qkv_splits || !splits) return -1;
+  *qkv_splits = sg::gemm_qkv_splits(M, N, K, precision, (size_t)-1);
+  *splits = sg::gemm_splits(M, N, K, precision);
   return 0;
 }
 

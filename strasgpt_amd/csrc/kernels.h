@@ -175,10 +175,11 @@ void gemm(const GemmParams& p, int epilogue, int precision, int splits, hipStrea
 // 4 K steps per split. Llama-3.2-1B shape, 8 rows: 22.4 -> 13.6 us (the fused
 // GEMM has 48 blocks of 64 x 64). Above 128 rows the GEMM splits when that
 // fills one round of 64 x 128 tiles at two per CU (MXFP4 MoE shape at 256
-// rows: 3 splits, 35.2 -> 29.2 us with the sums).
-int gemm_qkv_splits(int M, int N, int K, size_t ws_floats);
+// rows: 3 splits, 35.2 -> 29.2 us with the sums). The precision decides which
+// tiles run (gemm), and with them the count.
+int gemm_qkv_splits(int M, int N, int K, int precision, size_t ws_floats);
 // Split-K factor that fills the CUs for an M x N output (1: no split).
-int gemm_splits(int M, int N, int K);
+int gemm_splits(int M, int N, int K, int precision);
 
 // -------------------------------------------------------- elementwise --
 void embed(const int* tok, int T, const uint16_t* table, int d, float* x, hipStream_t s);

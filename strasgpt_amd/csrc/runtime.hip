@@ -643,7 +643,7 @@ int residual_gemm(Dev* D, const uint16_t* a_hi, const uint16_t* a_lo, int lda,
   g.N = N;
   g.K = K;
   g.ldc = N;
-  int splits = sg::gemm_splits(T, N, K);
+  int splits = sg::gemm_splits(T, N, K, D->precision);
   if (splits > 1 && (size_t)splits * T > (size_t)D->ws_splits * D->ws_rows)
     splits = (int)std::max<size_t>(1, (size_t)D->ws_splits * D->ws_rows / T);  // the workspace's rows of d
   Prof pr(D, cls, (double)N * K * 2, 2.0 * T * N * K);
@@ -709,7 +709,7 @@ void layer_prefill(Dev* D, int l, int T, const uint16_t* next_norm) {
   g.ctx = D->ctx;
   g.kv_bf16 = D->kv_bf16;
   g.kstage = D->kv_bf16 ? D->kstage : nullptr;
-  const int sp = sg::gemm_qkv_splits(T, D->qkv_rows, D->d, (size_t)D->ws_splits * D->ws_rows * D->d);
+  const int sp = sg::gemm_qkv_splits(T, D->qkv_rows, D->d, D->precision, (size_t)D->ws_splits * D->ws_rows * D->d);
   {
     Prof pr(D, K_QKV_GEMM, (double)D->qkv_rows * d * 2, 2.0 * M * D->qkv_rows * d);
     if (sp > 1) {

@@ -9,11 +9,14 @@ from strasgpt_amd import _paths, synth
 pytestmark = pytest.mark.skipif(not os.path.exists(_paths.hip_lib()), reason="library not built")
 
 
-def gemm_splits(M, N, K):
+BF16X2, BF16 = 0, 1
+
+
+def gemm_splits(M, N, K, precision=BF16X2):
     """(splits as the QKV projection, as the O or down projection)."""
     from strasgpt_amd import runtime as rt
     qkv, other = ctypes.c_int(), ctypes.c_int()
-    assert rt.lib().strasgpt_kbench_gemm_splits(M, N, K, ctypes.byref(qkv), ctypes.byref(other)) == 0
+    assert rt.lib().strasgpt_kbench_gemm_splits(M, N, K, precision, ctypes.byref(qkv), ctypes.byref(other)) == 0
     return qkv.value, other.value
 
 
@@ -36,3 +39,30 @@ def test_thin_row_splits_fill_the_cus(name):
         assert n > 1 and (qkv[0] + 63) // 64 * n >= 128, (M, qkv, n)
         as_qkv, as_o = gemm_splits(M, *o)
         assert as_qkv == as_o, (M, o)
+
+
+@pytest.mark.parametrize("name,qkv,o,down", [("llama3.2-1b", 8, 8, 8), ("qwen3-4b", 6, 8, 8), ("llama3.1-8b", 6, 8, 8),
+                                             ("mistral-small-24b", 6, 7, 8), ("moe-mxfp4", 7, 8, None)])
+def test_single_bf16_few_rows_square_counts(name, qkv, o, down):
+    """Single bf16 operands at up to 32 rows run the square tiles and take
+    the counts made for them, not the thin tiles' (fewer) ones."""
+    shapes = projections(synth.shape(name))
+    for M in (9, 16, 31, 32):
+        assert gemm_splits(M, *shapes[0], BF16)[0] == qkv
+        assert gemm_splits(M, *shapes[1], BF16)[1] == o
+        if down:
+            assert gemm_splits(M, *shapes[2], BF16)[1] == down
+
+
+@pytest.mark.parametrize("precision", [BF16X2, BF16])
+@pytest.mark.parametrize("name", sorted(synth.PRESETS))
+def test_forced_tile_square_counts(name, precision, monkeypatch):
+    """With a tile shape forced the square tiles run at any length: a split
+    QKV projection of 33 to 128 rows has one round of 64 x 128 tiles (two per
+    CU, at least three quarters of the 512 slots)."""
+    monkeypatch.setenv("STRASGPT_GEMM_TILE", "64x128x64")
+    qkv = projections(synth.shape(name))[0]
+    for M in (33, 45, 64, 65, 96, 128):
+        n, _ = gemm_splits(M, *qkv, precision)
+        tiles = (qkv[0] + 127) // 128 * ((M + 63) // 64)
+        assert n == 1 or 384 <= tiles * n <= 512, (M, n, tiles)
