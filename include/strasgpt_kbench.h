@@ -55,6 +55,11 @@ int strasgpt_kbench_sort_desc(const uint32_t* keys, int n, uint32_t* keys_out, i
  * workspace without bound, splits as the O or down projection. */
 int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, int* qkv_splits, int* splits);
 
+/* Slots per tile (16, 32 or 64) that the grouped expert GEMMs take for
+ * `slots` (token, expert) pairs over `experts` experts; -1 for invalid
+ * arguments (host arithmetic). */
+int strasgpt_kbench_moe_slot_tile(int slots, int experts);
+
 #ifdef __cplusplus
 }
 #endif

@@ -162,6 +162,10 @@ extern "C" int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, i
   return 0;
 }
 
+extern "C" int strasgpt_kbench_moe_slot_tile(int slots, int experts) {
+  return slots < 1 || experts < 1 ? -1 : sg::moe_slot_tile(slots, experts);
+}
+
 static int mxfp4_decode_hook(const uint8_t* codes, const uint8_t* scales, int nblocks, float* out,
                              int bf16_tiles) {
   if (nblocks <= 0 || !codes || !scales || !out) return -1;

@@ -875,9 +875,9 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(MoeGemmParams p) {
 //   E8M0 scales are DMA'd once per block and converted to fp32 a step ahead;
 // * each wave converts the codes of its own weight rows straight into its
 //   MFMA B operands (hardware FP4 conversion to packed bf16 pairs, exact),
-//   so no decoded tile goes through LDS: BM = 64 slots (for experts that
-//   average at least 24, so that one tile covers most of them and their
-//   weights stream once; group_gemm3_kernel takes fewer) x QBR rows x 64 K
+//   so no decoded tile goes through LDS: BM = 64 slots (for experts with
+//   so many that one tile covers most of them and their weights stream
+//   once, moe_slot_tile; group_gemm3_kernel takes fewer) x QBR rows x 64 K
 //   per step, 4 BM / 16
 //   QFR MFMAs per wave (each wave: all BM slots x QFR 16-row fragments;
 //   a 2 x 2 split of the waves, half the A stage each but twice the code
@@ -1244,8 +1244,9 @@ __global__ __launch_bounds__(256, 2) void group_gemm2_kernel(MoeGemmParams p) {
 //   tokens                  8        21        64       128       192
 //   64 (32, 64 slots)   77, 47    98, 51   105, 54   115, 61   142, 80
 //   128 (16, 32 slots)  63, 33    73, 37    82, 43   107, 61   132, 71
-// From 24 slots per expert on the 64-slot tile of group_gemm2_kernel is the
-// better one (its two stages of 128 would leave one block per CU). The A stage holds rows of 256 bytes, chunk ch of row r at
+// For more slots per expert (moe_slot_tile) the 64-slot tile of
+// group_gemm2_kernel is the better one (its two stages of 128 would leave one
+// block per CU). The A stage holds rows of 256 bytes, chunk ch of row r at
 // ch ^ (r & 15); the code stage rows of 64 bytes, block b of row r at
 // b ^ ((r >> 2) & 3): fragment reads meet no bank conflicts.
 template <int BM>
@@ -1557,13 +1558,16 @@ void moe_gather_split(const MoeGemmParams& p, hipStream_t s) {
   HIP_CHECK(hipGetLastError());
 }
 
-// Slots per tile of the grouped GEMM by the experts' average: 64 from 24
-// slots on (one tile covers most experts, so their weights stream once);
-// below, 16 (a tile of few slots reads little but its weights), with 32
-// between 12 and 18, where most experts need two tiles of 16 and one of 32.
-// Gate/up + down at the MXFP4 MoE shape, us with 16, 32 and 64 slots: 8 slots
-// on average 125, 148, 183; 12.5: 166, 163, 193; 16: 172, 169, 199; 24: 203,
-// 217, 223; 28: 231, 222, 226; 32: 250, 266, 239; 50: 340, 344, 302.
+// Slots per tile of the grouped GEMM by the experts' average. Few slots: 16
+// (a tile reads little but its weights). 32 from 12 to 28, where most experts
+// need two tiles of 16 and one of 32; from 29 on more and more of them need
+// two of 32, and three of 16 hold them with less padding. 64 from 37 on (one
+// tile covers most experts, so their weights stream once). Gate/up + down in
+// prompts of the MXFP4 MoE shape, us, mean of three prompts' routings:
+//   average   8    12    18    24    28    30    32    36    38    44    64
+//   16      146   174   190   206   225   233   236   249   260   284   386
+//   32      162   171   180   204   221   243   247   261   272   298   392
+//   64      195   206   216   230   240   241   245   252   255   269   363
 // STRASGPT_MOE_TILE=16|32|64 forces one (tests).
 int moe_slot_tile(int slots, int E) {
   const char* v = getenv("STRASGPT_MOE_TILE");
@@ -1572,7 +1576,7 @@ int moe_slot_tile(int slots, int E) {
     if (t != 16 && t != 32 && t != 64) ST_DIE("STRASGPT_MOE_TILE must be 16, 32 or 64");
     return t;
   }
-  return slots >= 24 * E ? 64 : slots >= 12 * E && slots < 18 * E ? 32 : 16;
+  return slots >= 37 * E ? 64 : slots >= 12 * E && slots < 29 * E ? 32 : 16;
 }
 
 void moe_group_gemm(const MoeGemmParams& p, hipStream_t s) {

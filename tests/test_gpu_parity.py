@@ -823,9 +823,9 @@ def test_logits_window_and_chunking(model_dir):
 
 
 def test_moe_grouped_gemm_slot_tiles(model_dir, monkeypatch):
-    """The grouped prefill GEMM with 32- and with 64-slot tiles
-    (STRASGPT_MOE_TILE; 64 is taken when the experts average 24 slots or
-    more): the same logits to fp32 rounding, both against the oracle."""
+    """The grouped prefill GEMM with 16-, 32- and 64-slot tiles
+    (STRASGPT_MOE_TILE; by default the experts' average decides): each against
+    the oracle, and the same logits bit for bit."""
     rt = runtime()
     d = model_dir("tiny-moe-long")
     shp = synth.shape("tiny-moe-long")
@@ -833,7 +833,7 @@ def test_moe_grouped_gemm_slot_tiles(model_dir, monkeypatch):
     ol = oracle_model(d, 4).predict(prompt)
     got = {}
     with rt.Transformer(d) as t:
-        for tile in ("32", "64"):
+        for tile in ("16", "32", "64"):
             monkeypatch.setenv("STRASGPT_MOE_TILE", tile)
             t.reset()
             got[tile] = t.predict(prompt)
@@ -841,6 +841,7 @@ def test_moe_grouped_gemm_slot_tiles(model_dir, monkeypatch):
             log(f"tiny-moe-long, {tile}-slot tiles: max |logit error| {err:.3g}")
             np.testing.assert_allclose(got[tile], ol, rtol=RTOL, atol=ATOL)
     # the slot tiling does not change any product's K order
+    np.testing.assert_array_equal(got["16"], got["64"])
     np.testing.assert_array_equal(got["32"], got["64"])
 
 
@@ -849,7 +850,7 @@ def test_moe_grouped_gemm_slot_tiles(model_dir, monkeypatch):
 def test_moe_tiny_against_oracle(name, model_dir):
     """MXFP4 MoE decoder: tokens identical to the oracle (the build's own
     restatement; no reference counterpart exists). The long prompt runs the
-    grouped prefill GEMMs with several 32-slot tiles per expert; mid-moe
+    grouped prefill GEMMs with several slot tiles per expert; mid-moe
     runs the decode kernels on 2880-wide rows (90 MXFP4 blocks) with top-4."""
     rt = runtime()
     d = model_dir(name)

@@ -66,3 +66,18 @@ def test_forced_tile_square_counts(name, precision, monkeypatch):
         n, _ = gemm_splits(M, *qkv, precision)
         tiles = (qkv[0] + 127) // 128 * ((M + 63) // 64)
         assert n == 1 or 384 <= tiles * n <= 512, (M, n, tiles)
+
+
+@pytest.mark.parametrize("experts", [8, 32])
+def test_moe_slot_tile_by_average(experts, monkeypatch):
+    """Slots per expert tile at both sides of every change of the rule; the
+    environment variable forces one."""
+    from strasgpt_amd import runtime as rt
+    tile = rt.lib().strasgpt_kbench_moe_slot_tile
+    for average, want in ((1, 16), (11, 16), (12, 32), (24, 32), (28, 32), (29, 16), (32, 16), (36, 16), (37, 64),
+                          (64, 64)):
+        assert tile(average * experts, experts) == want, average
+    assert tile(12 * experts - 1, experts) == 16 and tile(37 * experts - 1, experts) == 16
+    for forced in (16, 32, 64):
+        monkeypatch.setenv("STRASGPT_MOE_TILE", str(forced))
+        assert tile(24 * experts, experts) == forced
