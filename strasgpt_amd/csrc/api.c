@@ -40,7 +40,7 @@ float* transformer_logits_malloc(transformer_t* transformer, size_t logits_count
 /* In pieces of at least 512 KiB, on up to 8 threads: one thread touching
  * fresh pages copies at a fraction of the memory's rate. Inside a parallel
  * region (the reference driver's team) the nested region is one thread. */
-void host_copy(void* dst, const void* src, size_t n) {
+void st_host_copy(void* dst, const void* src, size_t n) {
   const size_t piece = (size_t)512 << 10;
   const int most = omp_get_max_threads() < 8 ? omp_get_max_threads() : 8;
   const size_t parts = n / piece < (size_t)most ? n / piece : (size_t)most;

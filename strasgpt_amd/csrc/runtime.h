@@ -39,7 +39,7 @@ int sg_profile_read(transformer_t* t, int kernel_class, transformer_kernel_stat_
 int sg_kernel_rate(transformer_t* t, int kernel_class, int reps, double* avg_us, double* bytes);
 
 /* memcpy, by several threads for large n (api.c) */
-void host_copy(void* dst, const void* src, size_t n);
+void st_host_copy(void* dst, const void* src, size_t n);
 
 #ifdef __cplusplus
 }

@@ -1101,7 +1101,7 @@ bool argmax_to(Dev* D, const float* row, bool log_seq, bool bump_pos, bool embed
 
 // `bytes` of device memory to the caller's pageable `dst`, through the two
 // halves of the pinned staging buffer: while one half is filled over PCIe
-// the other is copied out, by several threads where that pays (host_copy).
+// the other is copied out, by several threads where that pays (st_host_copy).
 // The runtime's own pageable copy runs one thread, and most of a large copy
 // is that thread taking the page faults of a buffer not yet touched: 50 MB
 // of logits in 4.9 ms, staged 2.1 ms.
@@ -1121,7 +1121,7 @@ void copy_out(Dev* D, char* dst, const char* src, size_t bytes) {
   for (size_t c = 0; c < chunks; c++) {
     const size_t at = c * kStageHalf, n = std::min(kStageHalf, bytes - at);
     HIP_CHECK(hipEventSynchronize(D->stage_ev[c % 2]));
-    host_copy(dst + at, D->h_stage + (c % 2) * kStageHalf, n);
+    st_host_copy(dst + at, D->h_stage + (c % 2) * kStageHalf, n);
     if (c + 2 < chunks) fill(c + 2);
   }
 }
