@@ -964,9 +964,19 @@ void layer_prefill_rows(Dev* D, int l, int T) {
 // planes (hi + lo + lo2 = the fp32 value exactly, so every product is exact
 // in the fp32 accumulator): the smallest plane's product is stored, the
 // other two's added to it. 777 rows of a 16032 x 4096 matrix: a GEMV per row
-// 20.7 ms, the GEMMs 0.43 ms. 16 rows (two multi-row GEMVs against the
-// GEMMs), us: 16032 x 4096 72 : 83, 128256 x 2048 192 : 362, 25120 x 2880
-// 94 : 95; 24 rows 108 : 88, 288 : 375, 141 : 101.
+// 20.7 ms, the GEMMs 0.43 ms. The GEMMs take over after two multi-row GEMVs
+// (of 8 rows; of 4 where 8 do not fit: d = 5120), GEMVs : GEMMs in us:
+//   rows             8           9          16          17          32
+//    16032 x 4096    36 :  62    65 :  62    73 :  62   101 :  63   146 :  65
+//    33504 x 2880    48 :  95    83 :  95    94 :  96   130 :  93   190 :  99
+//    37984 x 2560    43 :  85    81 :  86    87 :  87   126 :  87   176 :  92
+//   128256 x 2048   102 : 247   180 : 248   201 : 252   277 : 254   393 : 264
+//   151936 x 2560   136 : 361   252 : 366   281 : 371   391 : 385   555 : 403
+//   201088 x 2880   203 : 524   374 : 530   404 : 538   580 : 543   835 : 571
+//     6528 x 5120    39 :  68    56 :  68    77 :  69    95 :  70   155 :  74
+//   131072 x 5120   407 : 520   607 : 522   817 : 524  1015 : 528  1643 : 550
+// The rule is off only at 9 to 12 rows of the small d = 5120 matrix (10 to
+// 12 us) and at 10 to 16 rows of the 16032 x 4096 one (up to 10 us).
 void classifier(Dev* D, int T, int lc) {
   const uint16_t* w = D->tied ? W16(D, W_EMB) : W16(D, W_OUT);
   float* x = D->x + (size_t)(T - lc) * D->d;
