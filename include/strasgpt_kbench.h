@@ -60,6 +60,11 @@ int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, int* qkv_spl
  * arguments (host arithmetic). */
 int strasgpt_kbench_moe_slot_tile(int slots, int experts);
 
+/* Key ranges that the prefill attention splits `queries` queries over `keys`
+ * keys (theirs among them) into, with scratch without bound: 1 = none; -1 for
+ * invalid arguments (host arithmetic). */
+int strasgpt_kbench_attention_ranges(int q_heads, int head_dim, int queries, int keys);
+
 #ifdef __cplusplus
 }
 #endif

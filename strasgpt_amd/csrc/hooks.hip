@@ -166,6 +166,19 @@ extern "C" int strasgpt_kbench_moe_slot_tile(int slots, int experts) {
   return slots < 1 || experts < 1 ? -1 : sg::moe_slot_tile(slots, experts);
 }
 
+extern "C" int strasgpt_kbench_attention_ranges(int q_heads, int head_dim, int queries, int keys) {
+  if (q_heads < 1 || head_dim < 1 || queries < 1 || keys < queries) return -1;
+  float scratch;  // (only its presence is looked at)
+  sg::AttnParams p{};
+  p.q_heads = q_heads;
+  p.hd = head_dim;
+  p.T = queries;
+  p.keys = keys;
+  p.partial = &scratch;
+  p.partial_floats = (size_t)-1;
+  return sg::attention_prefill_ranges(p);
+}
+
 static int mxfp4_decode_hook(const uint8_t* codes, const uint8_t* scales, int nblocks, float* out,
                              int bf16_tiles) {
   if (nblocks <= 0 || !codes || !scales || !out) return -1;

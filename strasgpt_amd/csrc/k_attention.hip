@@ -1252,16 +1252,23 @@ void attention_split_rows(const float* kcache, const float* vcache, uint16_t* kh
   HIP_CHECK(hipGetLastError());
 }
 
-// Key ranges of a split-bf16 prefill launch of nqb query blocks per head:
-// where those leave most of the 512 block slots (two per CU) empty and there
-// are at least 16 tiles of 32 keys, as many ranges of at least 4 tiles as
-// fill the slots (up to 16). Prompts from an empty cache stay whole (few tiles,
-// or query blocks enough); 23, 45 and 91 queries of 32 heads after 4000 keys:
-// 167 -> 36, 36 and 44 us with the combining kernel.
-int prefill_ranges(const AttnParams& p, int nqb) {
+// Split bf16: 32 queries per wave (128 per block) when such blocks give 2 per CU.
+static bool prefill_wide(int T, int q_heads) { return (long)((T + 2 * PQ - 1) / (2 * PQ)) * q_heads >= 512; }
+
+// Where the (query block, head) pairs leave most of the 512 block slots (two
+// per CU) empty and there are at least 16 tiles of 32 keys: as many ranges of
+// at least 4 tiles as fill the slots (up to 16). 23, 45 and 91 queries of 32
+// heads of 128 after 4000 keys: 167 -> 36, 36 and 44 us with the combining
+// kernel; a whole prompt from an empty cache has few enough pairs where the
+// heads are few (512 queries of 8 heads of 128: 27 -> 20). Heads of 64 and
+// less with 128 pairs and more stay whole below 20 tiles: the walk is short
+// there and the ranges' partial results many (512 queries of 16 heads of 64:
+// 16.8 us whole, 18.4 in 4 ranges; 640 queries, 20 tiles: 19.5 and 18.9).
+int attention_prefill_ranges(const AttnParams& p) {
+  if (!p.partial || prefill_wide(p.T, p.q_heads)) return 1;
   const int tiles = (p.keys + kX3Keys - 1) / kX3Keys;
-  const long blocks = (long)nqb * p.q_heads;
-  if (!p.partial || blocks >= 256 || tiles < 16) return 1;
+  const long blocks = (long)((p.T + PQ - 1) / PQ) * p.q_heads;
+  if (blocks >= 256 || tiles < 16 || (p.hd <= 64 && blocks >= 128 && tiles < 20)) return 1;
   long r = std::min<long>({512 / blocks, 16, tiles / 4});
   while (r > 1 && (size_t)r * p.T * p.q_heads * (p.hd + 2) > p.partial_floats) r--;
   return (int)std::max<long>(r, 1);
@@ -1275,12 +1282,11 @@ void attention_prefill_variant(const AttnParams& p, int variant, hipStream_t s) 
   if (variant < 0 || variant > 3) ST_DIE("prefill attention variant is 0 (split bf16), 1 (fp32), 2 or 3");
   if (variant == 1 && p.kv_bf16) ST_DIE("the fp32 prefill attention kernel reads an fp32 KV cache only");
   const bool fp32 = variant == 1;
-  // split bf16: 32 queries per wave when 128-query blocks give 2 per CU
-  const bool wide = variant == 3 || (variant == 0 && (long)((p.T + 2 * PQ - 1) / (2 * PQ)) * p.q_heads >= 512);
+  const bool wide = variant == 3 || (variant == 0 && prefill_wide(p.T, p.q_heads));
   const int nqb = (p.T + (wide ? 2 * PQ : PQ) - 1) / (wide ? 2 * PQ : PQ);
   // x3: (heads, query blocks), longest ranges of every head first; fp32: (query blocks, heads)
   const dim3 grid = fp32 ? dim3(nqb, p.q_heads) : dim3(p.q_heads, nqb);
-  const int ranges = variant == 0 && !wide ? prefill_ranges(p, nqb) : 1;
+  const int ranges = variant == 0 ? attention_prefill_ranges(p) : 1;
   const dim3 gsplit(p.q_heads, nqb, ranges), gmerge((p.T * p.q_heads * p.hd / 4 + 255) / 256);
   switch (p.hd) {
 #define PREFILL_CASE(HD)                                                                         \

@@ -280,6 +280,8 @@ struct AttnParams {
   unsigned* counters;    // [kv_heads], zero between launches
 };
 void attention_prefill(const AttnParams& p, hipStream_t s);
+// Key ranges that the split-bf16 form of it takes (1: whole).
+int attention_prefill_ranges(const AttnParams& p);
 // variant 0: split-bf16 matrix cores (16 or 32 queries per wavefront by the
 // grid size), 1: fp32 matrix cores, 2 / 3: split bf16 with 16 / 32 queries
 void attention_prefill_variant(const AttnParams& p, int variant, hipStream_t s);
