@@ -69,23 +69,31 @@ def test_short_prompts_continued(kv, tmp_path):
 @pytest.mark.parametrize("kv", ["fp32", "bf16"])
 def test_short_prompts_after_long_context(kv, tmp_path):
     """Few queries after a context of 16 key tiles and more: the prefill
-    attention split over key ranges (an empty last range; a range that some
-    queries of a block see nothing of; 2 to 8 rows with fp32 outputs), against
-    the same prompt in one call, which is not split. Bound as above."""
+    attention split over key ranges (empty last ranges: 65 tiles in 16 ranges
+    of 5; a range that some queries of a block see nothing of; 2 to 8 rows with
+    fp32 outputs), against the same prompt in one call, whose query blocks fill
+    the GPU and are not split (both as the launch rule says). Bound as above."""
     from strasgpt_amd import runtime as rt
-    shp = synth.dataclasses.replace(SHAPES[1], name="thin-context", ctx=900)
+    shp = synth.dataclasses.replace(SHAPES[1], name="thin-context", heads=32, kv_heads=8, ctx=2100)
     d = str(tmp_path / shp.name)
     synth.write_model(shp, d, seed=11)
-    prompt = synth.prompt_tokens(shp.vocab, 889, PROMPT_SEED)
+    prompt = synth.prompt_tokens(shp.vocab, 2059, PROMPT_SEED)
+
+    def ranges(queries, keys):
+        return rt.lib().strasgpt_kbench_attention_ranges(shp.heads, shp.head_dim, queries, keys)
+
     with rt.Transformer(d) as t:
         if kv == "bf16":
             t.set_kv_cache_format(rt.KV_BF16)
-        for cuts in ((600, 120, 45, 3, 9), (511, 2), (700, 90, 64)):
+        for cuts, split in (((600, 120, 45, 3, 9), (1, 5, 5, 6, 6)), ((511, 2), (1, 4)),
+                            ((700, 90, 64), (1, 6, 6)), ((2050, 9), (1, 16))):
+            assert ranges(sum(cuts), sum(cuts)) == 1
             t.reset()
             want = t.predict(prompt[:sum(cuts)])[0]
             t.reset()
             at = 0
-            for n in cuts:
+            for n, r in zip(cuts, split):
+                assert ranges(n, at + n) == r
                 got = t.predict(prompt[at:at + n])[0]
                 at += n
             err = float(np.abs(got - want).max())
