@@ -85,7 +85,7 @@ def test_short_prompts_after_long_context(kv, tmp_path):
     with rt.Transformer(d) as t:
         if kv == "bf16":
             t.set_kv_cache_format(rt.KV_BF16)
-        for cuts, split in (((600, 120, 45, 3, 9), (1, 5, 5, 6, 6)), ((511, 2), (1, 4)),
+        for cuts, split in (((600, 120, 45, 3, 9), (1, 5, 6, 6, 6)), ((511, 2), (1, 4)),
                             ((700, 90, 64), (1, 6, 6)), ((2050, 9), (1, 16))):
             assert ranges(sum(cuts), sum(cuts)) == 1
             t.reset()
