@@ -22,7 +22,6 @@ def test_large_logits_reach_the_caller(vocab, rows, tmp_path):
     |value|: a misplaced or stale piece is off by the values themselves), in
     fresh, unaligned and pinned buffers bit for bit the same, nothing beside
     them written; a second prompt through the same halves likewise."""
-    import torch
     from oracle import oracle as orc
     from strasgpt_amd import runtime as rt
     shp = synth.ModelShape("copy", 64, 96, 1, 4, 1, 32, vocab, 500000.0, 1e-5, 100, 4, ctx=104, std=0.25)
@@ -30,6 +29,10 @@ def test_large_logits_reach_the_caller(vocab, rows, tmp_path):
     synth.write_model(shp, d, seed=11)
     oracle = orc.OracleModel(d, threads=16)
     n = rows * vocab
+    hip = rt.lib()  # (its HIP runtime's functions are found through it)
+    address = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(address), ctypes.c_size_t(4 * (n + 6)), 0) == 0
+    pinned = np.ctypeslib.as_array(ctypes.cast(address, ctypes.POINTER(ctypes.c_float)), (n + 6,))
     with rt.Transformer(d) as t:
         def into(buffer, at, prompt):
             t.reset()
@@ -47,14 +50,10 @@ def test_large_logits_reach_the_caller(vocab, rows, tmp_path):
             print(f"[logits copy] {rows} x {vocab}: max |error| {err:.3g}", flush=True)
             np.testing.assert_allclose(got.reshape(rows, vocab), want, rtol=2e-2, atol=1e-3)
             assert (fresh[:3] == -7.0).all() and (fresh[3 + n:] == -7.0).all()
-            pinned = torch.full((n + 6,), -7.0, pin_memory=True)
-            into(pinned.data_ptr(), 3, prompt)
-            whole = pinned.numpy()
-            np.testing.assert_array_equal(whole[3:3 + n], got)
-            assert (whole[:3] == -7.0).all() and (whole[3 + n:] == -7.0).all()
-            np.testing.assert_array_equal(t_predict(t, prompt, rows).reshape(-1), got)
-
-
-def t_predict(t, prompt, rows):
-    t.reset()
-    return t.predict(prompt, rows)
+            pinned[:] = -7.0
+            into(address.value, 3, prompt)
+            np.testing.assert_array_equal(pinned[3:3 + n], got)
+            assert (pinned[:3] == -7.0).all() and (pinned[3 + n:] == -7.0).all()
+            t.reset()
+            np.testing.assert_array_equal(t.predict(prompt, rows).reshape(-1), got)
+    assert hip.hipHostFree(address) == 0
