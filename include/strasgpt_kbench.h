@@ -60,6 +60,10 @@ int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, int* qkv_spl
  * arguments (host arithmetic). */
 int strasgpt_kbench_moe_slot_tile(int slots, int experts);
 
+/* Wavefronts per block (4, 6 or 8) of the few-token expert down projection
+ * onto N outputs; -1 for invalid arguments (host arithmetic). */
+int strasgpt_kbench_moe_down_waves(int N, int tokens);
+
 /* Key ranges that the prefill attention splits `queries` queries over `keys`
  * keys (theirs among them) into, with scratch without bound: 1 = none; -1 for
  * invalid arguments (host arithmetic). */

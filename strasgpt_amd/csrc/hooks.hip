@@ -166,6 +166,10 @@ extern "C" int strasgpt_kbench_moe_slot_tile(int slots, int experts) {
   return slots < 1 || experts < 1 ? -1 : sg::moe_slot_tile(slots, experts);
 }
 
+extern "C" int strasgpt_kbench_moe_down_waves(int N, int tokens) {
+  return N < 1 || tokens < 1 ? -1 : sg::moe_down_waves(N, tokens);
+}
+
 extern "C" int strasgpt_kbench_attention_ranges(int q_heads, int head_dim, int queries, int keys) {
   if (q_heads < 1 || head_dim < 1 || queries < 1 || keys < queries) return -1;
   float scratch;  // (only its presence is looked at)

@@ -99,6 +99,8 @@ void moe_route_logits(const float* x, const uint16_t* norm_w, float eps, const u
 bool moe_route_logits_supported(int E, int topk, int d);
 void moe_gemv_swiglu(const MoeGemvParams& p, hipStream_t s);
 void moe_gemv_down(const MoeGemvParams& p, hipStream_t s);
+// Wavefronts per block of it (4, 6 or 8).
+int moe_down_waves(int N, int tokens);
 // Prefill MoE: slots grouped by expert, then grouped MXFP4 GEMMs.
 // order[offs[e] .. offs[e+1]) lists the slots routed to expert e in
 // increasing order (offs has E + 1 entries).
