@@ -11,12 +11,14 @@
 //     of probabilities in index order exceeds the coin.
 //
 // Differences from the sequential host code are in summation order only:
-// the softmax sum, the top-p running sum and the index-order running sum
-// are formed from fixed-order partial sums (deterministic, but rounded
-// differently), so a draw can differ from the reference's only when the
-// coin or top_p lies within that rounding of a boundary. Equal
-// probabilities rank by index (the radix sort below is stable), as a
-// stable sort of the reference's index-ordered array ranks them. The coin stream, the
+// the softmax sum and the renormalisation's double sum, and without a top-k of
+// at most 1024 the top-p and the index-order running sums too, are formed from
+// fixed-order partial sums (deterministic, but rounded differently), so a
+// draw can differ from the reference's only when the coin or top_p lies within
+// that rounding of a boundary. (A top-k of at most 1024 adds both running sums
+// one probability after the other, as the reference does.) Equal probabilities
+// rank by index, as a stable sort of the reference's index-ordered array ranks
+// them. The coin stream, the
 // penalty and every per-element operation (division by the temperature,
 // expf, division by the sum, multiplication by the float inverse of the
 // double sum) are the reference's.

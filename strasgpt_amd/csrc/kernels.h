@@ -84,8 +84,8 @@ struct MoeGemvParams {
   const float* weight;     // [tokens][topk] routing weights (down-proj only)
   int tokens, topk, N, K;
   float* y;                // SWIGLU: [tokens*topk][N]; DOWN: y[t][n] += routed sum
-  // Decode (one token, E <= 64): router logits [E] instead of expert /
-  // weight; each block selects the top-k itself.
+  // SWIGLU in decode (one token, E <= 64): router logits [E] instead of
+  // expert; each block selects the top-k itself.
   const float* logits;
   int E;
   // SWIGLU with logits: the selection, for the down projection ([topk], or null)

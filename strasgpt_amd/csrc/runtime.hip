@@ -378,8 +378,8 @@ bool ffn_moe(Dev* D, int l, int T) {
   const double d = D->d, H = D->H, k = D->topk;
   const bool fused = T == 1 && sg::moe_route_logits_supported(D->E, D->topk, D->d);
   if (fused) {
-    // decode: RMSNorm + router logits in one launch; the expert kernels
-    // select the top-k from the logits themselves
+    // decode: RMSNorm + router logits in one launch; the gate/up kernel
+    // selects the top-k from the logits itself and writes it for the down one
     Prof pr(D, K_ROUTE, (double)D->E * d * 2, 2.0 * D->E * d);
     sg::moe_route_logits(D->x, W16(D, W_FFN_NORM, l), D->eps, W16(D, W_ROUTER, l), D->E, D->d, D->moe_logits,
                          D->xn, s);
@@ -395,7 +395,7 @@ bool ffn_moe(Dev* D, int l, int T) {
   }
   if (T >= kMoeGroupedMinTokens) {
     // prefill: slots grouped by expert, each expert's weights read once per
-    // 32-slot tile (MFMA GEMMs), then the routed sum in top-k order
+    // slot tile (MFMA GEMMs), then the routed sum in top-k order
     const int n = T * D->topk;
     const double used = std::min((double)n, (double)D->E);
     sg::moe_group(D->moe_sel, n, D->E, D->moe_offs, D->moe_order, s);

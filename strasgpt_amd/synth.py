@@ -114,8 +114,8 @@ TINY: Dict[str, ModelShape] = {
     # (512 rows: 2 row tiles; QKV 12, O 4, gate/up 16, down 4 column tiles).
     "mid-dense": ModelShape("mid-dense", 1024, 2048, 1, 8, 8, 128, 512, 500000.0, 1e-5,
                             512, 4, ctx=600, untied=True, std=0.02),
-    # A short prompt on wide rows: the QKV prefill GEMM takes the split-K
-    # form with the separate epilogue (8 rows, 4 splits).
+    # A short prompt on wide rows: the QKV prefill GEMM is split over K (8
+    # rows, 4 splits), and the QK-norm/RoPE kernel adds the partial sums.
     "small-m": ModelShape("small-m", 1024, 2048, 2, 8, 2, 128, 512, 500000.0, 1e-5,
                           8, 6, ctx=64, untied=True, std=0.02),
     # FFN rows longer than one LDS stage of the decode GEMV (64 KiB of

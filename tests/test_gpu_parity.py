@@ -120,11 +120,10 @@ def test_gemm_tile_orders(model_dir, monkeypatch):
 
 
 def test_small_prompt_split_gemms(model_dir, monkeypatch):
-    """Prompts of at most 32 rows run the QKV GEMM split over K (partial
-    sums, then an epilogue kernel that adds them in split order and writes
-    q and the key / value cache rows): prefill logits and greedy tokens
-    against the oracle, and a 40-row prompt (the fused epilogue) agrees
-    too. (Dense prompts of at most 8 rows take the multi-row GEMVs unless
+    """Short prompts run the QKV GEMM split over K (partial sums, which the
+    QK-norm/RoPE kernel adds in split order on its way to q and the key / value
+    cache rows): prefill logits and greedy tokens against the oracle, at 8 and
+    at 40 rows. (Dense prompts of at most 8 rows take the multi-row GEMVs unless
     STRASGPT_PREFILL_ROWS=0, which this test sets.)"""
     monkeypatch.setenv("STRASGPT_PREFILL_ROWS", "0")
     rt = runtime()
