@@ -55,10 +55,11 @@ int strasgpt_kbench_sort_desc(const uint32_t* keys, int n, uint32_t* keys_out, i
  * workspace without bound, splits as the O or down projection. */
 int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, int* qkv_splits, int* splits);
 
-/* Slots per tile (16, 32 or 64) that the grouped expert GEMMs take for
- * `slots` (token, expert) pairs over `experts` experts; -1 for invalid
- * arguments (host arithmetic). */
-int strasgpt_kbench_moe_slot_tile(int slots, int experts);
+/* Slots per tile (16, 32 or 64) that a grouped expert GEMM of N outputs (pair:
+ * gate and up of N each) over K inputs takes for `slots` (token, expert) pairs
+ * over `experts` experts, and its K per step; -1 for invalid arguments (host
+ * arithmetic). */
+int strasgpt_kbench_moe_slot_tile(int slots, int experts, int N, int K, int pair, int* k_step);
 
 /* Wavefronts per block (4, 6 or 8) of the few-token expert down projection
  * onto N outputs; -1 for invalid arguments (host arithmetic). */

@@ -162,8 +162,11 @@ extern "C" int strasgpt_kbench_gemm_splits(int M, int N, int K, int precision, i
   return 0;
 }
 
-extern "C" int strasgpt_kbench_moe_slot_tile(int slots, int experts) {
-  return slots < 1 || experts < 1 ? -1 : sg::moe_slot_tile(slots, experts);
+extern "C" int strasgpt_kbench_moe_slot_tile(int slots, int experts, int N, int K, int pair, int* k_step) {
+  if (slots < 1 || experts < 1 || N < 1 || K < 64 || !k_step) return -1;
+  const sg::MoeTile t = sg::moe_slot_tile(slots, experts, N, K, pair != 0);
+  *k_step = t.step;
+  return t.slots;
 }
 
 extern "C" int strasgpt_kbench_moe_down_waves(int N, int tokens) {

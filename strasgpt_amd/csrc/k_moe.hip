@@ -877,8 +877,7 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(MoeGemmParams p) {
 //   MFMA B operands (hardware FP4 conversion to packed bf16 pairs, exact),
 //   so no decoded tile goes through LDS: BM = 64 slots (for experts with
 //   so many that one tile covers most of them and their weights stream
-//   once, moe_slot_tile; group_gemm3_kernel takes fewer) x QBR rows x 64 K
-//   per step, 4 BM / 16
+//   once) or 32 (moe_slot_tile) x QBR rows x 64 K per step, 4 BM / 16
 //   QFR MFMAs per wave (each wave: all BM slots x QFR 16-row fragments;
 //   a 2 x 2 split of the waves, half the A stage each but twice the code
 //   conversions, measured slower). Every wave reads the whole A stage, so wider blocks read A
@@ -886,8 +885,8 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(MoeGemmParams p) {
 //   the work, but its grid of half as many blocks (at two per CU, 75 KiB of
 //   LDS) leaves a partial last round at the 256-token prefill and loses
 //   there (228 vs 193 us for the gate/up pair); it wins at 2048 tokens
-//   (927 vs 1018 us). QBR = 128: ~73 KiB of LDS at K = 2880, two blocks
-//   per CU.
+//   (927 vs 1018 us). QBR = 128: ~73 KiB of LDS at K = 2880 with 64 slots,
+//   two blocks per CU, ~50 KiB with 32, three.
 // * the grid is laid out per XCD (see the kernel).
 // Each step issues exactly QAI A + QBI code DMA instructions per wave
 // (indexes past the last step are clamped to it and never read), so the
@@ -1031,8 +1030,7 @@ __device__ __forceinline__ void group_store(const MoeGemmParams& p, const f32x4 
     }
 }
 
-// BM slots per block (64: experts that average enough slots that one tile
-// covers most of them, so each expert's weights stream once).
+// BM slots per block (32 or 64).
 template <bool DUAL, int BM>
 __global__ __launch_bounds__(256, 2) void group_gemm2_kernel(MoeGemmParams p) {
   using QL = QLds<BM>;
@@ -1244,9 +1242,9 @@ __global__ __launch_bounds__(256, 2) void group_gemm2_kernel(MoeGemmParams p) {
 //   tokens                  8        21        64       128       192
 //   64 (32, 64 slots)   77, 47    98, 51   105, 54   115, 61   142, 80
 //   128 (16, 32 slots)  63, 33    73, 37    82, 43   107, 61   132, 71
-// For more slots per expert (moe_slot_tile) the 64-slot tile of
-// group_gemm2_kernel is the better one (its two stages of 128 would leave one
-// block per CU). The A stage holds rows of 256 bytes, chunk ch of row r at
+// For more slots per expert group_gemm2_kernel is the better one
+// (moe_slot_tile; 64 slots in two stages of 128 would leave one block per CU).
+// The A stage holds rows of 256 bytes, chunk ch of row r at
 // ch ^ (r & 15); the code stage rows of 64 bytes, block b of row r at
 // b ^ ((r >> 2) & 3): fragment reads meet no bank conflicts.
 template <int BM>
@@ -1561,25 +1559,48 @@ void moe_gather_split(const MoeGemmParams& p, hipStream_t s) {
   HIP_CHECK(hipGetLastError());
 }
 
-// Slots per tile of the grouped GEMM by the experts' average. Few slots: 16
-// (a tile reads little but its weights). 32 from 12 to 28, where most experts
-// need two tiles of 16 and one of 32; from 29 on more and more of them need
-// two of 32, and three of 16 hold them with less padding. 64 from 37 on (one
-// tile covers most experts, so their weights stream once). Gate/up + down in
-// prompts of the MXFP4 MoE shape, us, mean of three prompts' routings:
-//   average   8    12    18    24    28    30    32    36    38    44    64
-//   16      146   174   190   206   225   233   236   249   260   284   386
-//   32      162   171   180   204   221   243   247   261   272   298   392
-//   64      195   206   216   230   240   241   245   252   255   269   363
-// STRASGPT_MOE_TILE=16|32|64 forces one (tests).
-int moe_slot_tile(int slots, int E) {
+// Tile of the pipelined grouped GEMM by the experts' average of slots and by
+// the width of the code rows. Few slots: 16 in steps of 128
+// (group_gemm3_kernel): a tile reads little but its weights. More slots would
+// read them again for every 16; what that costs depends on the L2 channels
+// (16 of 256 bytes) that a column of code rows, K / 2 bytes apart, is spread
+// over: on all 16, no other tile wins before 64 slots do at 37; on fewer, 32
+// slots in steps of 64 (group_gemm2_kernel) win from about 9000 channels / K
+// slots on. Measured for 15 pairs of widths (512 to 7168, 8 to 128 experts, 4
+// to 96 slots on average); gate/up, us, 16 slots : 32 (64) : 64:
+//   K, experts (channels)   8              16              24              40
+//   2880,  32 (16)       91 : 110 : 127 109 : 124 : 143 130 : 148 : 148 169 : 186 : 175
+//   2560,  40 (16)       49 :  61 :  68  55 :  63 :  73  66 :  67 :  77  86 :  83 :  85
+//   3072,  64 (8)        65 :  79 :  86  73 :  83 :  97  88 :  90 : 106 125 : 123 : 131
+//   5120,  64 (8)       151 : 170 : 301 192 : 186 : 321 236 : 227 : 345 363 : 323 : 394
+//   2048, 128 (4)        63 :  68 :  86  83 :  83 :  97 105 :  93 : 109 149 : 124 : 133
+//   4096, 128 (2)       276 : 274 : 302 367 : 310 : 335 486 : 345 : 366 714 : 510 : 420
+// 64 slots take over at 24 for 2 channels and at 64 for 4 and 8, and only where
+// two blocks fit a CU's LDS (K to about 4600: at 5120 one block, as above).
+// Wide GEMMs over all channels take 32 slots in steps of 128 from 12 to 28:
+// MXFP4 MoE shape, gate/up + down in prompts of random tokens, 16 : 32 slots at
+// 12 170 : 166 us, at 18 185 : 175, at 24 203 : 201, at 28 221 : 217, at 30
+// 230 : 239 (with other routings of these widths 6% more to 6% less).
+// STRASGPT_MOE_TILE=16|32|64 forces the slots (tests).
+MoeTile moe_slot_tile(int slots, int E, int N, int K, bool dual) {
+  int channels = 16;
+  for (int stride = K / 2 / 256; K / 2 % 256 == 0 && stride % 2 == 0 && channels > 1; stride /= 2) channels /= 2;
+  const MoeTile few{16, 128}, mid{32, channels == 16 ? 128 : 64}, many{64, 64};
   const char* v = getenv("STRASGPT_MOE_TILE");
   if (v && *v) {
     const int t = atoi(v);
     if (t != 16 && t != 32 && t != 64) ST_DIE("STRASGPT_MOE_TILE must be 16, 32 or 64");
-    return t;
+    return t == 16 ? few : t == 32 ? mid : many;
   }
-  return slots >= 37 * E ? 64 : slots >= 12 * E && slots < 29 * E ? 32 : 16;
+  const int runs = dual ? 2 : 1;
+  const bool pair = 2 * (QLds<64>::sc + runs * q_scale_run(QBR / runs, K / 32)) <= 160 * 1024;
+  const double average = (double)slots / E;
+  if (channels == 16) {
+    if (average >= 37) return pair ? many : MoeTile{32, 64};
+    return average >= 12 && average < 29 && N >= 2560 && K >= 2560 ? mid : few;
+  }
+  if (pair && average >= (channels <= 2 ? 24 : 64)) return many;
+  return average >= std::min(37, 9000 * channels / K) ? mid : few;
 }
 
 void moe_group_gemm(const MoeGemmParams& p, hipStream_t s) {
@@ -1589,8 +1610,10 @@ void moe_group_gemm(const MoeGemmParams& p, hipStream_t s) {
   if (moe_group_gemm2_ok(p)) {
     const bool dual = p.blocks2 != nullptr;
     const int nb = p.K / 32, runs = dual ? 2 : 1;
-    const int bm = moe_slot_tile(p.slots, p.E);
-    const size_t shm = (bm == 64 ? QLds<64>::sc : bm == 32 ? QwLds<32>::sc : QwLds<16>::sc) + (size_t)runs * q_scale_run(QBR / runs, nb);
+    const MoeTile tile = moe_slot_tile(p.slots, p.E, p.N, p.K, dual);
+    const int bm = tile.slots;
+    const int stages = bm == 64 ? QLds<64>::sc : bm == 16 ? QwLds<16>::sc : tile.step == 64 ? QLds<32>::sc : QwLds<32>::sc;
+    const size_t shm = (size_t)stages + (size_t)runs * q_scale_run(QBR / runs, nb);
     const int cols = dual ? QBR / 2 : QBR;
     // slot tiles: an upper bound (the counts are on the device), rounded to
     // whole rounds of the XCDs (the kernel's per-XCD layout)
@@ -1603,12 +1626,14 @@ void moe_group_gemm(const MoeGemmParams& p, hipStream_t s) {
   } while (0)
     if (dual) {
       if (bm == 64) GG(group_gemm2_kernel, true, 64);
-      else if (bm == 32) GG(group_gemm3_kernel, true, 32);
-      else GG(group_gemm3_kernel, true, 16);
+      else if (bm == 16) GG(group_gemm3_kernel, true, 16);
+      else if (tile.step == 64) GG(group_gemm2_kernel, true, 32);
+      else GG(group_gemm3_kernel, true, 32);
     } else {
       if (bm == 64) GG(group_gemm2_kernel, false, 64);
-      else if (bm == 32) GG(group_gemm3_kernel, false, 32);
-      else GG(group_gemm3_kernel, false, 16);
+      else if (bm == 16) GG(group_gemm3_kernel, false, 16);
+      else if (tile.step == 64) GG(group_gemm2_kernel, false, 32);
+      else GG(group_gemm3_kernel, false, 32);
     }
 #undef GG
     HIP_CHECK(hipGetLastError());

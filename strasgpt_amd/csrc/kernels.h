@@ -125,8 +125,11 @@ struct MoeGemmParams {
   uint16_t *y_hi, *y_lo;
 };
 void moe_group_gemm(const MoeGemmParams& p, hipStream_t s);
-// Slots per tile (16, 32 or 64) of its pipelined kernels.
-int moe_slot_tile(int slots, int E);
+// Tile of its pipelined kernels: slots (16, 32 or 64) and K per step.
+struct MoeTile {
+  int slots, step;
+};
+MoeTile moe_slot_tile(int slots, int E, int N, int K, bool dual);
 // a_hi/a_lo[i] = split of the A row of slot order[i] (a[order[i] / topk] when
 // a_per_token, else a[order[i]]), i < slots (for an A in expert order when
 // the previous GEMM could not write its planes).

@@ -68,19 +68,34 @@ def test_forced_tile_square_counts(name, precision, monkeypatch):
         assert n == 1 or 384 <= tiles * n <= 512, (M, n, tiles)
 
 
-@pytest.mark.parametrize("experts", [8, 32])
-def test_moe_slot_tile_by_average(experts, monkeypatch):
-    """Slots per expert tile at both sides of every change of the rule; the
-    environment variable forces one."""
+FEW, MANY = (16, 128), (64, 64)
+MID, MID64 = (32, 128), (32, 64)
+
+
+@pytest.mark.parametrize("N,K,pair,changes", [
+    (2880, 2880, 1, [(1, FEW), (12, MID), (29, FEW), (37, MANY)]),  # code rows over all 16 L2 channels, wide
+    (1280, 2560, 1, [(1, FEW), (37, MANY)]), (4096, 1536, 0, [(1, FEW), (37, MANY)]),
+    (6000, 4800, 1, [(1, FEW), (12, MID), (29, FEW), (37, MID64)]),  # one block of 64 slots per CU
+    (1024, 3072, 1, [(1, FEW), (23, MID64), (64, MANY)]), (1536, 5120, 1, [(1, FEW), (14, MID64)]),  # 8 channels
+    (2048, 1024, 0, [(1, FEW), (37, MID64), (64, MANY)]),
+    (768, 2048, 1, [(1, FEW), (17, MID64), (64, MANY)]), (1024, 6144, 1, [(1, FEW), (5, MID64)]),  # 4
+    (1536, 4096, 1, [(1, FEW), (4, MID64), (24, MANY)])])  # 2
+def test_moe_slot_tile(N, K, pair, changes, monkeypatch):
+    """The grouped GEMM's tile at both sides of every change of the rule, with
+    few and many experts; the environment variable forces the slots."""
     from strasgpt_amd import runtime as rt
-    tile = rt.lib().strasgpt_kbench_moe_slot_tile
-    for average, want in ((1, 16), (11, 16), (12, 32), (24, 32), (28, 32), (29, 16), (32, 16), (36, 16), (37, 64),
-                          (64, 64)):
-        assert tile(average * experts, experts) == want, average
-    assert tile(12 * experts - 1, experts) == 16 and tile(37 * experts - 1, experts) == 16
+    step = ctypes.c_int()
+
+    def tile(slots, experts):
+        return rt.lib().strasgpt_kbench_moe_slot_tile(slots, experts, N, K, pair, ctypes.byref(step)), step.value
+
+    for experts in (8, 128):
+        for (at, want), (end, _) in zip(changes, changes[1:] + [(400, None)]):
+            assert tile(at * experts, experts) == want, (at, experts)
+            assert tile(end * experts - 1, experts) == want, (end, experts)
     for forced in (16, 32, 64):
         monkeypatch.setenv("STRASGPT_MOE_TILE", str(forced))
-        assert tile(24 * experts, experts) == forced
+        assert tile(8, 8)[0] == forced
 
 
 @pytest.mark.parametrize("heads,hd,queries,keys,ranges", [
