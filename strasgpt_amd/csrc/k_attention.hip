@@ -1261,14 +1261,16 @@ static bool prefill_wide(int T, int q_heads) { return (long)((T + 2 * PQ - 1) / 
 // heads of 128 after 4000 keys: 167 -> 36, 36 and 44 us with the combining
 // kernel; a whole prompt from an empty cache has few enough pairs where the
 // heads are few (512 queries of 8 heads of 128: 27 -> 20). Heads of 64 and
-// less with 128 pairs and more stay whole below 20 tiles: the walk is short
-// there and the ranges' partial results many (512 queries of 16 heads of 64:
-// 16.8 us whole, 18.4 in 4 ranges; 640 queries, 20 tiles: 19.5 and 18.9).
+// less with 96 pairs and more stay whole below 20 tiles: the walk is short
+// there, the ranges' partial results many, and there is one more launch (512
+// queries of 64-wide heads, whole and in 4 ranges: 8 heads 16.5 and 12.9 us, 16
+// heads 16.8 and 18.4; 640 queries of 16, 20 tiles: 19.5 and 18.9; a 520-token
+// prompt of 6 layers with 14 heads 766 and 778 us).
 int attention_prefill_ranges(const AttnParams& p) {
   if (!p.partial || prefill_wide(p.T, p.q_heads)) return 1;
   const int tiles = (p.keys + kX3Keys - 1) / kX3Keys;
   const long blocks = (long)((p.T + PQ - 1) / PQ) * p.q_heads;
-  if (blocks >= 256 || tiles < 16 || (p.hd <= 64 && blocks >= 128 && tiles < 20)) return 1;
+  if (blocks >= 256 || tiles < 16 || (p.hd <= 64 && blocks >= 96 && tiles < 20)) return 1;
   long r = std::min<long>({512 / blocks, 16, tiles / 4});
   while (r > 1 && (size_t)r * p.T * p.q_heads * (p.hd + 2) > p.partial_floats) r--;
   return (int)std::max<long>(r, 1);

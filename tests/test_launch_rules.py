@@ -102,10 +102,11 @@ def test_moe_slot_tile(N, K, pair, changes, monkeypatch):
     (32, 128, 45, 4045, 16), (32, 128, 448, 4448, 2), (32, 128, 449, 4449, 1),  # blocks fill the slots
     (32, 128, 45, 480, 1), (32, 128, 45, 481, 4),  # 15 and 16 tiles
     (16, 64, 512, 512, 1), (24, 64, 512, 512, 1), (16, 64, 608, 608, 1), (16, 64, 640, 640, 3),  # 16, 19, 20 tiles
-    (8, 64, 512, 512, 4), (16, 128, 512, 512, 4), (15, 64, 512, 512, 4),  # fewer pairs; longer steps
+    (8, 64, 512, 512, 4), (11, 64, 512, 512, 4), (12, 64, 512, 512, 1), (14, 64, 520, 520, 1),  # 88, 96 and 126 pairs
+    (16, 128, 512, 512, 4),  # longer steps
     (64, 128, 8192, 8192, 1), (1, 16, 1, 1, 1)])
 def test_prefill_attention_ranges(heads, hd, queries, keys, ranges):
-    """Both sides of each line of the rule. Short walks of 128 pairs and more
+    """Both sides of each line of the rule. Short walks of 96 pairs and more
     with heads of 64 stay whole: their ranges were the slower form."""
     from strasgpt_amd import runtime as rt
     assert rt.lib().strasgpt_kbench_attention_ranges(heads, hd, queries, keys) == ranges
