@@ -222,11 +222,14 @@ __global__ __launch_bounds__(kPick) void sample_pick_kernel(SampleParams p) {
 }
 
 // ----------------------------------------------------------- small top-k --
-// top_k of at most kTopMax (the usual case) needs no sort of the vocabulary:
-// three launches instead of seventeen. Bound by their launches and chains of
-// barriers, not by bytes (V floats read and written twice): V = 128256,
-// k = 50, 225 -> 32 us a draw, of which the full sort's picking kernel
-// took 121 (one block walking the whole vocabulary) and the sort 81.
+// top_k of at most kTopMax (the usual case) needs no sort of the
+// vocabulary: three launches instead of seventeen. Bound by their launches and
+// chains of barriers, not by bytes (V floats read and written twice):
+// V = 128256, k = 50, 225 -> 29 us a draw, of which the full sort's picking
+// kernel took 121 (one block walking the whole vocabulary) and the sort 81;
+// k = 1024 with a top-p 235 -> 130, at V = 32000 107 -> 83. The worst case is a
+// vocabulary of equal probabilities, all of them candidates of the one drawing
+// block: 236 us, the full sort 207 and 14 launches more.
 // * scale (above): penalty, temperature, block maxima;
 // * exp: expf, block sums, and each block's candidates: the elements in the
 //   eighth-octave bins of expf down to the bin that holds the block's k-th
@@ -370,10 +373,29 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kST / WAVE; i++) sum += red[i];
-  // larger probability first, then the lower index: distinct keys
-  auto item = [&](unsigned c) -> unsigned long long {
-    const float q = __uint_as_float(p.keys_sorted[c]) / sum;
-    return ((unsigned long long)__float_as_uint(q) << 32) | (unsigned)~p.vals_sorted[c];
+  // Every candidate's key (larger probability first, then the lower index:
+  // distinct) to f(valid, key), by all lanes of a wavefront together, kU
+  // candidates a thread in flight: near-uniform distributions make candidates
+  // of the whole vocabulary, and one at a time each pass over 128256 of them
+  // waited 125 latencies.
+  auto each = [&](auto f) {
+    constexpr int kU = 8;
+    for (unsigned c0 = 0; c0 < total; c0 += kU * kPick) {
+      unsigned kb[kU];
+      int vi[kU];
+#pragma unroll
+      for (int u = 0; u < kU; u++) {
+        const unsigned c = min(c0 + u * kPick + tid, total - 1);
+        kb[u] = p.keys_sorted[c];
+        vi[u] = p.vals_sorted[c];
+      }
+#pragma unroll
+      for (int u = 0; u < kU; u++) {
+        if (c0 + u * kPick >= total) break;
+        const float q = __uint_as_float(kb[u]) / sum;
+        f(c0 + u * kPick + tid < total, ((unsigned long long)__float_as_uint(q) << 32) | (unsigned)~vi[u]);
+      }
+    }
   };
 
   // Radix selection: 12-bit digits from the top until what lies at or above
@@ -388,10 +410,20 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
     for (int b = tid; b < kTopBins; b += kPick) hist[b] = 0u;
     if (tid == 0) above[kPick] = 0u;
     __syncthreads();
-    for (unsigned c = tid; c < total; c += kPick) {
-      const unsigned long long x = item(c);
-      if (shift == 64 || (x >> shift) == prefix) atomicAdd(&hist[(unsigned)(x >> low) & ((1u << bits) - 1u)], 1u);
-    }
+    each([&](bool valid, unsigned long long x) {
+      const bool in = valid && (shift == 64 || (x >> shift) == prefix);
+      const unsigned b = (unsigned)(x >> low) & ((1u << bits) - 1u);
+      const unsigned long long m = __ballot(in);
+      if (!m) return;
+      const int first = __ffsll((long long)m) - 1;
+      // one addition where the wavefront's digits agree (ties: 64 additions
+      // to one address are done one after the other)
+      if (__ballot(in && b == (unsigned)__builtin_amdgcn_readlane((int)b, first)) == m) {
+        if (lane == first) atomicAdd(&hist[b], (unsigned)__popcll(m));
+      } else if (in) {
+        atomicAdd(&hist[b], 1u);
+      }
+    });
     __syncthreads();
     constexpr int PER = kTopBins / kPick;
     unsigned mine = 0u;
@@ -429,38 +461,51 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
     if (over + bin_s <= (unsigned)kTopCap || shift == 0) break;
     __syncthreads();  // prefix_s, above_s and bin_s are read before the next digit's
   }
-  for (unsigned c = tid; c < total; c += kPick) {
-    const unsigned long long x = item(c);
-    if ((x >> shift) >= prefix) {
+  each([&](bool valid, unsigned long long x) {
+    if (valid && (x >> shift) >= prefix) {
       const unsigned at = atomicAdd(&got, 1u);
       if (at < (unsigned)kTopCap) key[at] = x;
     }
-  }
+  });
   __syncthreads();
   const int n0 = (int)min(got, (unsigned)kTopCap);
   sort_desc_lds(key, sorted, n0);
 
-  // The cut: the first k, or fewer where the running sum reaches top_p.
-  const int kact = min((int)k, n0);
-  if (tid < WAVE) {
-    int n = kact;
-    if (p.top_p > 0.0f && p.top_p <= 1.0f) {
-      float cum = 0.0f;
-      bool found = false;
-      for (int at = 0; at < kact && !found; at += WAVE) {
-        const float v = at + lane < kact ? __uint_as_float((unsigned)(sorted[at + lane] >> 32)) : 0.0f;
-        const int m = min(WAVE, kact - at);
-        for (int j = 0; j < m; j++) {
-          cum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-          if (cum >= p.top_p) {
-            n = at + j + 1;
-            found = true;
-            break;
-          }
+  // Running sums of value[0 .. n) one after the other (the reference's
+  // order), by one thread: 32 values requested while 32 are added. (A wavefront
+  // that took its lanes' values in turn and tested each sum needed 50 ns for
+  // each: 1024 kept tokens of 32000 130 us a draw, now 83.)
+  float *value = (float*)hist, *cum = value + kTopMax;
+  auto running_sums = [&](int n) {
+    __syncthreads();
+    if (tid == 0) {
+      constexpr int B = 32;
+      float x[B], c = 0.0f;
+#pragma unroll
+      for (int u = 0; u < B; u++) x[u] = value[u];
+      for (int at = 0; at < n; at += B) {  // (past n: values never looked at)
+        float y[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) y[u] = value[min(at + B, kTopMax - B) + u];
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+          c += x[u];
+          cum[at + u] = c;
         }
+#pragma unroll
+        for (int u = 0; u < B; u++) x[u] = y[u];
       }
     }
-    if (lane == 0) kept_s = n;
+    __syncthreads();
+  };
+
+  // The cut: the first k, or fewer where the running sum reaches top_p.
+  const int kact = min((int)k, n0);
+  if (tid == 0) kept_s = kact;
+  if (p.top_p > 0.0f && p.top_p <= 1.0f) {
+    if (tid < kact) value[tid] = __uint_as_float((unsigned)(sorted[tid] >> 32));
+    running_sums(kact);
+    if (tid < kact && cum[tid] >= p.top_p) atomicMin(&kept_s, tid + 1);
   }
   __syncthreads();
   const int n = kept_s;
@@ -509,26 +554,13 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
     for (int r = tid; r < n; r += kPick) key[r] = (sorted[r] << 32) | (sorted[r] >> 32);
     __syncthreads();
     sort_desc_lds(key, sorted, n);
-    if (tid < WAVE) {
-      float cdf = 0.0f;
-      bool found = false;
-      for (int at = 0; at < n && !found; at += WAVE) {
-        const unsigned long long x = at + lane < n ? sorted[at + lane] : 0ull;
-        const float wl = __uint_as_float((unsigned)x) * inv;
-        const int idx = (int)~(unsigned)(x >> 32), m = min(WAVE, n - at);
-        for (int j = 0; j < m; j++) {
-          const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wl), j));
-          const int pick = __builtin_amdgcn_readlane(idx, j);
-          cdf += w;
-          if (w > 0.0f && coin < cdf) {
-            if (lane == 0) best = pick;
-            found = true;
-            break;
-          }
-        }
-      }
-    }
+    const float w = tid < n ? __uint_as_float((unsigned)sorted[tid]) * inv : 0.0f;
+    if (tid < n) value[tid] = w;
+    if (tid == 0) kept_s = n;  // (its value is in n)
+    running_sums(n);
+    if (tid < n && w > 0.0f && coin < cum[tid]) atomicMin(&kept_s, tid);
     __syncthreads();
+    if (tid == 0 && kept_s < n) best = (int)~(unsigned)(sorted[kept_s] >> 32);
   }
   if (tid == 0) {
     const int tok = best < V ? best : V - 1;  // rounding fallback, as the reference's
