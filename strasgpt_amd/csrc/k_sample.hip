@@ -227,9 +227,9 @@ __global__ __launch_bounds__(kPick) void sample_pick_kernel(SampleParams p) {
 // chains of barriers, not by bytes (V floats read and written twice):
 // V = 128256, k = 50, 225 -> 29 us a draw, of which the full sort's picking
 // kernel took 121 (one block walking the whole vocabulary) and the sort 81;
-// k = 1024 with a top-p 235 -> 130, at V = 32000 107 -> 83. The worst case is a
+// k = 1024 with a top-p 235 -> 122, at V = 32000 107 -> 78. The worst case is a
 // vocabulary of equal probabilities, all of them candidates of the one drawing
-// block: 236 us, the full sort 207 and 14 launches more.
+// block: 233 us, the full sort 207 and 14 launches more.
 // * scale (above): penalty, temperature, block maxima;
 // * exp: expf, block sums, and each block's candidates: the elements in the
 //   eighth-octave bins of expf down to the bin that holds the block's k-th
@@ -380,6 +380,15 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
   // waited 125 latencies.
   auto each = [&](auto f) {
     constexpr int kU = 8;
+    auto keyed = [&](unsigned c, unsigned e, int index) {
+      const float q = __uint_as_float(e) / sum;
+      f(c < total, ((unsigned long long)__float_as_uint(q) << 32) | (unsigned)~index);
+    };
+    if (total <= (unsigned)kPick) {
+      const unsigned c = min((unsigned)tid, total - 1);
+      keyed(tid, p.keys_sorted[c], p.vals_sorted[c]);
+      return;
+    }
     for (unsigned c0 = 0; c0 < total; c0 += kU * kPick) {
       unsigned kb[kU];
       int vi[kU];
@@ -392,8 +401,7 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
 #pragma unroll
       for (int u = 0; u < kU; u++) {
         if (c0 + u * kPick >= total) break;
-        const float q = __uint_as_float(kb[u]) / sum;
-        f(c0 + u * kPick + tid < total, ((unsigned long long)__float_as_uint(q) << 32) | (unsigned)~vi[u]);
+        keyed(c0 + u * kPick + tid, kb[u], vi[u]);
       }
     }
   };
@@ -472,14 +480,16 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
   sort_desc_lds(key, sorted, n0);
 
   // Running sums of value[0 .. n) one after the other (the reference's
-  // order), by one thread: 32 values requested while 32 are added. (A wavefront
-  // that took its lanes' values in turn and tested each sum needed 50 ns for
-  // each: 1024 kept tokens of 32000 130 us a draw, now 83.)
+  // order), by one thread: 16 values requested while 16 are added, up to the
+  // 16 that hold the first sum that ends the walk (later ones are not written:
+  // whatever is there comes after it). (A wavefront that took its lanes' values
+  // in turn and tested each sum needed 50 ns for each: 1024 kept tokens of
+  // 32000 130 us a draw, now 78.)
   float *value = (float*)hist, *cum = value + kTopMax;
-  auto running_sums = [&](int n) {
+  auto running_sums = [&](int n, auto ends) {
     __syncthreads();
     if (tid == 0) {
-      constexpr int B = 32;
+      constexpr int B = 16;
       float x[B], c = 0.0f;
 #pragma unroll
       for (int u = 0; u < B; u++) x[u] = value[u];
@@ -492,6 +502,7 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
           c += x[u];
           cum[at + u] = c;
         }
+        if (ends(c)) break;
 #pragma unroll
         for (int u = 0; u < B; u++) x[u] = y[u];
       }
@@ -504,7 +515,7 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
   if (tid == 0) kept_s = kact;
   if (p.top_p > 0.0f && p.top_p <= 1.0f) {
     if (tid < kact) value[tid] = __uint_as_float((unsigned)(sorted[tid] >> 32));
-    running_sums(kact);
+    running_sums(kact, [&](float c) { return c >= p.top_p; });
     if (tid < kact && cum[tid] >= p.top_p) atomicMin(&kept_s, tid + 1);
   }
   __syncthreads();
@@ -557,7 +568,7 @@ __global__ __launch_bounds__(kPick) void sample_draw_kernel(SampleParams p, cons
     const float w = tid < n ? __uint_as_float((unsigned)sorted[tid]) * inv : 0.0f;
     if (tid < n) value[tid] = w;
     if (tid == 0) kept_s = n;  // (its value is in n)
-    running_sums(n);
+    running_sums(n, [&](float c) { return coin < c; });
     if (tid < n && w > 0.0f && coin < cum[tid]) atomicMin(&kept_s, tid);
     __syncthreads();
     if (tid == 0 && kept_s < n) best = (int)~(unsigned)(sorted[kept_s] >> 32);
